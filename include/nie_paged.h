@@ -346,6 +346,22 @@ int64_t nie_workspace_control_bytes(void);
 int nie_decode_last_path(void);
 
 /*
+ * The kernels that a bf16 decode call with the reference rounding runs, given
+ * the alignment and workspace that the MFMA kernels take (a host-only query;
+ * arguments as in nie_paged_decode_workspace_bytes).  device_planned: the call
+ * of nie_paged_decode_append_planned with these bounds (no host lengths).
+ * NIE_DECODE_KERNEL_NONE for other calls and invalid arguments.
+ */
+#define NIE_DECODE_KERNEL_NONE 0
+#define NIE_DECODE_KERNEL_PASSES 1 /* scores pass, P.V pass, sum */
+#define NIE_DECODE_KERNEL_FUSED 2  /* one launch, K and V straight into registers */
+#define NIE_DECODE_KERNEL_RING 3   /* one launch, K and V through an LDS ring */
+#define NIE_DECODE_KERNEL_SHORT 4  /* one launch, a sequence's splits in one workgroup */
+int nie_paged_decode_kernel(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
+                            int64_t block_size, int64_t max_seq_len, int64_t total_seq_len,
+                            const int32_t* host_seq_lens, int device_planned);
+
+/*
  * Workspace bytes needed by nie_paged_decode for a call with these
  * arguments (same meaning as there; host values), whose sequence lengths
  * have maximum max_seq_len and sum total_seq_len, and the same optional

@@ -68,6 +68,7 @@ EXPORTED_SYMBOLS = (
     "nie_set_decode_fused_spin",
     "nie_workspace_control_bytes",
     "nie_decode_last_path",
+    "nie_paged_decode_kernel",
     "nie_paged_decode_workspace_bytes",
     "nie_paged_decode_workspace_wanted",
     "nie_paged_decode",
@@ -135,6 +136,7 @@ _SIGNATURES = {
     "nie_set_decode_fused_spin": (_i32, [_i32]),
     "nie_workspace_control_bytes": (_i64, []),
     "nie_decode_last_path": (_i32, []),
+    "nie_paged_decode_kernel": (_i32, [_i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _i32]),
     "nie_paged_decode_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr]),
     "nie_paged_decode_workspace_wanted": (_i64, [_i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr]),
     "nie_paged_decode": (
@@ -379,6 +381,18 @@ def workspace_control_bytes() -> int:
 def decode_last_path() -> str:
     """Which kernels this thread's last decode call ran ("fused", "passes", ...)."""
     return DECODE_PATHS[load_library().nie_decode_last_path()]
+
+
+DECODE_KERNELS = ("none", "passes", "fused", "ring", "short")
+
+
+def decode_kernel(dtype: torch.dtype, q_heads: int, kv_heads: int, head_dim: int, block_size: int, batch: int,
+                  max_seq_len: int, total_seq_len: int, seq_lens_host=None, device_planned: bool = False) -> str:
+    """The kernels that a reference-rounding decode call with these arguments runs ("none": other calls)."""
+    lens = _host_seq_lens(seq_lens_host, batch)
+    return DECODE_KERNELS[load_library().nie_paged_decode_kernel(
+        dtype_code(dtype), batch, q_heads, kv_heads, head_dim, block_size, max_seq_len, total_seq_len,
+        _array_ptr(lens), int(device_planned))]
 
 
 def _check(rc: int, what: str) -> None:
