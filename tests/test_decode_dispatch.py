@@ -54,3 +54,41 @@ def test_forced_split_length_fits_the_ring(forced):
         assert kernel in ("passes", "fused", "ring")
         if kernel == "ring":
             assert forced * (q_heads // kv_heads) <= RING_SCORE_ROWS[head_dim]
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,lens,kernel", [
+    # the shares that one wave of the ring sums, against the sum's launch
+    (16, 1, 64, [100] * 7 + [4000], "passes"),  # 125 splits of 16 rows: 54.5 us on the ring, 17.3 here
+    (16, 1, 64, [1000] * 4, "passes"),
+    (8, 1, 128, [2000] * 4, "passes"),
+    (14, 2, 64, [2000] * 4, "passes"),
+    (64, 8, 128, [1000] * 4, "passes"),  # 32 splits of 2 tiles, 8 rows
+    (64, 8, 128, [1000] * 16, "ring"),  # 8 splits of 8 tiles
+    (32, 8, 128, [100] * 15 + [3000], "passes"),  # 63 splits of 3 tiles
+    (32, 8, 128, [1000] * 8 + [3000], "ring"),  # 32 splits of 6 tiles
+    (32, 8, 128, [30000], "passes"),
+    (24, 8, 128, [2047, 331, 1200, 77, 905, 1618], "ring"),
+    # against decode_fused_kernel's sum
+    (32, 8, 64, [1000] * 4, "fused"),  # 32 splits of 2 tiles
+    (32, 8, 64, [100] * 15 + [2000], "fused"),
+    (32, 8, 64, [2000] * 16, "ring"),  # 16 splits of 8 tiles
+    (32, 8, 64, [1000] * 8 + [3000], "fused"),  # 63 splits of 3 tiles
+    (32, 8, 64, [90] * 33, "ring"),  # 3 splits of 2 tiles
+    (32, 32, 64, [2000], "fused"),
+    (32, 32, 64, [600] * 16, "ring"),
+    (8, 8, 64, [3000] * 8, "fused"),  # 32 splits of 6 tiles
+    # a sequence's splits in one workgroup
+    (32, 8, 64, [17, 64, 129, 500], "short"),
+    (32, 8, 64, [17, 64, 129, 513], "fused"),
+    (32, 8, 64, [60] * 32, "short"),
+    (32, 8, 64, [60] * 33, "ring"),  # more (sequence, KV head) pairs than CUs
+])
+def test_kernel_of_host_planned_calls(q_heads, kv_heads, head_dim, lens, kernel):
+    assert _kernel(q_heads, kv_heads, head_dim, lens) == kernel
+
+
+def test_shapes_outside_the_one_launch_kernels():
+    assert _kernel(32, 8, 64, [500] * 4, block_size=8) == "passes"  # tiles over several blocks
+    assert _kernel(32, 1, 64, [500] * 4) == "none"  # 32 rows: the generic kernel
+    assert _kernel(8, 8, 32, [500] * 4) == "none"
+    assert _native.decode_kernel(torch.float32, 32, 8, 64, 16, 4, 500, 2000, seq_lens_host=[500] * 4) == "none"

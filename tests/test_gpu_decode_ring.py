@@ -15,18 +15,21 @@ from tests.test_gpu_decode_fused import (  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 DEV = torch.device("cuda:0")
+KERNEL = "ring"  # what every case but the last runs on
 
 CASES = {  # q_heads, kv_heads, head_dim, block_size, contexts
     # a split of one key, a whole tile, a whole step, one key past each
-    "edges64": (32, 8, 64, 16, [0, 15, 16, 31, 32, 47, 64, 700] + [1200] * 12),
+    "edges64": (32, 8, 64, 16, [0, 15, 16, 31, 32, 47, 64, 700] + [1190] * 14),
     "edges128": (32, 8, 128, 16, [0, 15, 16, 31, 32, 47, 64, 700] + [600] * 12),
-    "one_head_group": (4, 2, 64, 32, [3000, 33, 1024, 5]),
-    "single_kv_head": (16, 1, 64, 16, [1500, 40, 777]),  # 16 query rows, many splits
-    "group1_dim128": (8, 8, 128, 16, [2000, 15, 640, 100]),
-    "group8_dim128": (64, 8, 128, 64, [1000, 15, 640, 100]),
+    "four_head_group": (16, 4, 64, 32, [i % 97 for i in range(100)]),
+    "two_head_group": (4, 2, 128, 16, [1000, 33, 15, 777]),
+    "one_head_group": (2, 1, 128, 32, [1000, 33, 15, 777]),
+    "group1_dim128": (8, 8, 128, 16, [2000, 15, 640, 100, 1990, 1500, 1200]),
+    "group8_dim128": (64, 8, 128, 64, [700, 15, 640, 100] + [650] * 12),
     "group3": (24, 8, 128, 16, [2047, 331, 1200, 77, 905, 1618]),
-    "group12": (12, 1, 128, 32, [900, 31, 2048]),
-    "many_splits": (32, 8, 64, 16, [2490, 20, 100]),  # 78 splits: two polls, several rounds of the sum
+    "group12": (48, 4, 128, 32, [7 * i % 311 for i in range(100)]),
+    "group16": (64, 4, 128, 16, [800 - i for i in range(40)]),  # every query row of the tile
+    "many_splits": (32, 8, 64, 16, [7990, 20, 8000, 8000, 8000]),  # 63 splits: two polls, several rounds of the sum
     "longest_splits": (32, 8, 64, 16, [8100] * 16),  # 32 tiles: the scores fill their region
     "past_the_ring": (32, 8, 64, 16, [9000] * 16),  # longer: decode_fused_kernel
 }
@@ -52,6 +55,9 @@ def _run(name: str, append: str):
 
         rope = RopeScale(head_dim).tables(DEV, dtype, max(wl.seq_lens))
     dq = q.to(DEV)
+    kernel = _native.decode_kernel(dtype, q_heads, kv_heads, head_dim, block_size, len(contexts), max(wl.seq_lens),
+                                   sum(wl.seq_lens), seq_lens_host=list(wl.seq_lens))
+    assert kernel == ("fused" if name == "past_the_ring" else KERNEL), kernel
 
     def run():
         k, v = kc.to(DEV), vc.to(DEV)

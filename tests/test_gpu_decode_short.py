@@ -30,6 +30,7 @@ CASES = {  # q_heads, kv_heads, head_dim, block_size, contexts
 @pytest.fixture(autouse=True)
 def _cases(monkeypatch):
     monkeypatch.setattr(ring, "CASES", CASES)
+    monkeypatch.setattr(ring, "KERNEL", "short")
 
 
 @pytest.mark.parametrize("name", list(CASES))
