@@ -4,6 +4,7 @@ decision that the call itself takes), checked without a GPU."""
 from __future__ import annotations
 
 import os
+import random
 import subprocess
 import sys
 
@@ -92,3 +93,41 @@ def test_shapes_outside_the_one_launch_kernels():
     assert _kernel(32, 1, 64, [500] * 4) == "none"  # 32 rows: the generic kernel
     assert _kernel(8, 8, 32, [500] * 4) == "none"
     assert _native.decode_kernel(torch.float32, 32, 8, 64, 16, 4, 500, 2000, seq_lens_host=[500] * 4) == "none"
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,batch,bound,kernel", [
+    (32, 8, 64, 4, 512, "fused"),  # a captured step of short sequences
+    (32, 8, 64, 16, 2048, "fused"),  # any of 2,000 tokens each, and one of them among short ones
+    (32, 8, 64, 16, 11776, "fused"),
+    (16, 1, 64, 8, 1024, "passes"),
+    (64, 8, 128, 8, 2048, "passes"),
+    (32, 8, 128, 16, 3072, "passes"),
+    (32, 8, 128, 43, 1024, "passes"),  # tables of 215 items in two rounds of 128
+    (32, 8, 128, 4, 512, "ring"),
+    (16, 8, 128, 4, 1024, "ring"),
+])
+def test_kernel_of_device_planned_calls(q_heads, kv_heads, head_dim, batch, bound, kernel):
+    assert _kernel(q_heads, kv_heads, head_dim, batch=batch, bound=bound) == kernel
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(32, 8, 128), (16, 8, 128), (8, 8, 128), (32, 32, 128), (4, 2, 128),
+                                                       (24, 8, 128), (64, 8, 128), (32, 8, 64), (32, 32, 64), (40, 5, 64)])
+def test_device_planned_ring_holds_for_every_table(q_heads, kv_heads, head_dim):
+    """A device-planned call on the ring: whatever lengths within its bounds
+    the table is written for, the host-planned call of these lengths runs on
+    the ring or in one workgroup per sequence and head, too."""
+    rng = random.Random(5)
+    rings = 0
+    for _ in range(300):
+        batch, bound = rng.choice([1, 2, 3, 4, 6, 8, 12, 16, 24, 40, 43, 64, 100]), rng.choice([64, 128, 192, 256, 512, 1024, 1536])
+        if _kernel(q_heads, kv_heads, head_dim, batch=batch, bound=bound) != "ring":
+            continue
+        rings += 1
+        low = rng.choice([1, bound // 2, bound - 20])
+        lens = [rng.randint(low, bound) if rng.random() < rng.choice([0.1, 0.9]) else rng.randint(1, 32)
+                for _ in range(batch)]
+        lens[0] = rng.choice([bound, lens[0]])
+        if not _native.decode_plan_fits(torch.bfloat16, q_heads, kv_heads, head_dim, 16, lens):
+            continue  # (no table: planned on the device)
+        assert _kernel(q_heads, kv_heads, head_dim, lens) in ("ring", "short"), (batch, bound, lens)
+    assert rings or q_heads // kv_heads > 4

@@ -5,6 +5,7 @@ around the edges of its tiles, steps, splits and score regions."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -116,4 +117,62 @@ def test_back_to_back_calls():
     torch.cuda.synchronize()
     for i, out in enumerate(outs):
         assert _same_bits(out, single[i % len(runs)]), i
+    assert _control_regions_zero()
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,bound,kernel", [
+    (32, 8, 128, 512, "ring"), (16, 8, 128, 1024, "ring"), (24, 8, 128, 512, "ring"), (32, 8, 64, 512, "fused")])
+def test_replays_of_a_device_planned_call(q_heads, kv_heads, head_dim, bound, kernel):
+    """One captured launch, replayed with tables of even, ragged and skewed
+    lengths (and none): each replay equals the eager call planned from the
+    host lengths bit for bit, cache included."""
+    print(f"device-planned replays: {q_heads}/{kv_heads} x {head_dim}, bound {bound}", flush=True)
+    dtype, batch, bs = torch.bfloat16, 4, 16
+    assert _native.decode_kernel(dtype, q_heads, kv_heads, head_dim, bs, batch, bound, batch * bound,
+                                 device_planned=True) == kernel
+    wl = workloads.ragged([bound - 1] * batch, [1] * batch, seed=29, pool_factor=1.2, q_heads=q_heads,
+                          kv_heads=kv_heads, head_dim=head_dim, block_size=bs)
+    kc, vc = wl.pool(dtype)
+    q, k_new, v_new = (t.to(DEV) for t in wl.new_tokens(dtype))
+    tables = torch.from_numpy(wl.table_array()).to(DEV)
+    lens = torch.zeros(batch, dtype=torch.int32, device=DEV)
+    plan = torch.zeros(-(-_native.decode_plan_bytes() // 4), dtype=torch.int32, device=DEV)
+    k, v, out = kc.to(DEV), vc.to(DEV), torch.empty_like(q)
+    scale = head_dim**-0.5
+
+    def host_plan(host):
+        buf = np.zeros(plan.numel(), dtype=np.int32)
+        _native.write_decode_plan(buf.ctypes.data, buf.nbytes, dtype, q_heads, kv_heads, head_dim, bs,
+                                  np.asarray(host, dtype=np.int32), max(host), sum(host))
+        assert buf[0] > 0
+        return torch.from_numpy(buf).to(DEV)
+
+    lens.copy_(torch.tensor([bound] * batch, dtype=torch.int32))
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        call = _native.PreparedDecode(k, v, tables, lens, bound, batch * bound, q_heads, scale, device_plan=plan)
+        call.append_decode(q, k_new, v_new, 0, out)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call.append_decode(q, k_new, v_new, 0, out)
+    for host, table in [([bound] * batch, True), ([1, 17, 40, bound], True), ([bound - 1, 33, 250, 16], True),
+                        ([5, 100, 64, 31], True), ([bound, 3, 200, 77], False), ([1, 2, 1, 1], True)]:
+        with torch.cuda.stream(stream):
+            k.copy_(kc)
+            v.copy_(vc)
+            lens.copy_(torch.tensor(host, dtype=torch.int32))
+            plan.copy_(host_plan(host)) if table else plan.zero_()
+            graph.replay()
+            stream.synchronize()
+        k2, v2 = kc.to(DEV), vc.to(DEV)
+        want = torch.empty_like(q)
+        _native.PreparedDecode(k2, v2, tables, lens, max(host), sum(host), q_heads, scale,
+                               seq_lens_host=host).append_decode(q, k_new, v_new, 0, want)
+        torch.cuda.synchronize()
+        if table:
+            assert _same_bits(out, want), host
+        else:  # (other splits)
+            assert (out.float() - want.float()).abs().max().item() <= 2e-2
+        assert _same_bits(k, k2) and _same_bits(v, v2), host
     assert _control_regions_zero()
