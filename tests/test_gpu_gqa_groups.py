@@ -95,6 +95,56 @@ def test_unaligned_rows_run_on_the_generic_kernel(dtype):
     assert _err(got.cpu(), want) <= TOL[dtype]
 
 
+def _attention_64(q, keys, values, scale, last):
+    """q (n, heads, dim), key and value rows of each query head's KV head, in 64 bits."""
+    seen = torch.arange(keys.shape[0], device=DEV)[None, :] <= last[:, None]
+    out = torch.empty(q.shape, dtype=torch.float64, device=DEV)
+    for h in range(q.shape[1]):
+        k, v = (t[:, h * keys.shape[1] // q.shape[1]].double().contiguous() for t in (keys, values))
+        scores = (q[:, h].double() @ k.t().contiguous()) * scale
+        out[:, h] = torch.softmax(scores.masked_fill(~seen, -torch.inf), dim=-1) @ v
+    return out
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(6, 2, 64), (24, 8, 128), (14, 2, 128), (26, 2, 128)])
+@pytest.mark.parametrize("contexts,queries", [([4000, 15, 700, 2000], [1] * 4), ([0, 200, 1500], [300, 128, 77])])
+def test_fp32_is_as_exact_as_the_generic_kernel(q_heads, kv_heads, head_dim, contexts, queries):
+    """Relative error against 64 bits, of the MFMA kernels and of the generic
+    ones (rows at element alignment) on the same numbers, over three draws."""
+    print(f"group fp32 error {q_heads}/{kv_heads} d={head_dim} {queries}", flush=True)
+    total = {"mfma": 0.0, "generic": 0.0}
+    for seed in (3, 4, 5):
+        wl = workloads.ragged(contexts, queries, seed=seed, pool_factor=1.2, q_heads=q_heads, kv_heads=kv_heads,
+                              head_dim=head_dim)
+        kc, vc = (t.to(DEV) for t in wl.pool(torch.float32))
+        q = wl.new_tokens(torch.float32)[0].to(DEV)
+        tables = torch.from_numpy(wl.table_array()).to(DEV)
+        scale, lens = head_dim**-0.5, list(wl.seq_lens)
+        want, at = torch.empty(q.shape, dtype=torch.float64, device=DEV), 0
+        for b, (n, m) in enumerate(zip(lens, queries)):
+            pos = torch.arange(n, device=DEV)
+            slots = tables[b][pos // wl.block_size].long() * wl.block_size + pos % wl.block_size
+            keys, values = (t[0].reshape(-1, kv_heads, head_dim)[slots] for t in (kc, vc))
+            want[at : at + m] = _attention_64(q[at : at + m], keys, values, scale, pos[n - m :])
+            at += m
+        if max(queries) == 1:
+            call = _native.PreparedDecode(kc, vc, tables, torch.tensor(lens, dtype=torch.int32, device=DEV), max(lens),
+                                          sum(lens), q_heads, scale, seq_lens_host=lens)
+        else:
+            cu = np.concatenate([[0], np.cumsum(queries)]).astype(np.int64)
+            call = _native.PreparedPrefill(kc, vc, torch.from_numpy(cu).to(DEV),
+                                           torch.tensor(contexts, dtype=torch.int32, device=DEV), tables, sum(queries),
+                                           max(queries), max(lens), q_heads, scale, cu_seqlens_host=cu.tolist(),
+                                           context_lens_host=contexts)
+        off = torch.empty(q.numel() + 1, device=DEV)[1:].view(q.shape).copy_(q)  # 4 bytes off 16
+        for name, rows in (("mfma", q), ("generic", off)):
+            out = torch.empty_like(q)
+            call(rows, 0, out)
+            total[name] += ((out.double() - want).norm() / want.norm()).item()
+    print(f"  {total}", flush=True)
+    assert total["mfma"] <= total["generic"]
+
+
 @pytest.mark.parametrize("q_heads,head_dim", [(6, 64), (6, 128)])
 def test_device_planned_decode_equals_host_planned(q_heads, head_dim, rounding):  # noqa: F811
     dtype = torch.bfloat16
