@@ -572,6 +572,22 @@ int64_t nie_varlen_prefill_workspace_bytes(int64_t num_seqs, int64_t total_query
                                            const int64_t* host_cu_seqlens,
                                            const int32_t* host_context_lens);
 
+/*
+ * Where the workgroups of a prefill call on the MFMA kernels take their query
+ * tiles from (a host-only query; arguments as in
+ * nie_varlen_prefill_workspace_bytes): a table written on the host, the device
+ * lengths by the keys a tile sees (calls of few requests whose tiles are one
+ * piece each), or the device lengths in request order.  The results do not
+ * depend on it.  NIE_PREFILL_ORDER_NONE for other calls and invalid arguments.
+ */
+#define NIE_PREFILL_ORDER_NONE 0
+#define NIE_PREFILL_ORDER_TABLE 1
+#define NIE_PREFILL_ORDER_SORTED 2
+#define NIE_PREFILL_ORDER_REQUESTS 3
+int nie_varlen_prefill_order(int64_t num_seqs, int64_t total_query_tokens, int64_t max_query_len,
+                             int64_t max_seq_len, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
+                             const int64_t* host_cu_seqlens, const int32_t* host_context_lens);
+
 /* As nie_paged_decode_workspace_wanted, for nie_varlen_prefill. */
 int64_t nie_varlen_prefill_workspace_wanted(int64_t num_seqs, int64_t total_query_tokens,
                                             int64_t max_query_len, int64_t max_seq_len,

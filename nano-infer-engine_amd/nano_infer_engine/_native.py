@@ -78,6 +78,7 @@ EXPORTED_SYMBOLS = (
     "nie_paged_decode_append_planned",
     "nie_paged_decode_noalloc_max_bytes",
     "nie_paged_decode_append_noalloc",
+    "nie_varlen_prefill_order",
     "nie_varlen_prefill_workspace_bytes",
     "nie_varlen_prefill_workspace_wanted",
     "nie_varlen_prefill",
@@ -214,6 +215,7 @@ _SIGNATURES = {
             _ptr, _ptr,                      # host seq_lens, stream
         ],
     ),
+    "nie_varlen_prefill_order": (_i32, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr]),
     "nie_varlen_prefill_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr]),
     "nie_varlen_prefill_workspace_wanted": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr]),
     "nie_varlen_prefill": (
@@ -393,6 +395,18 @@ def decode_kernel(dtype: torch.dtype, q_heads: int, kv_heads: int, head_dim: int
     return DECODE_KERNELS[load_library().nie_paged_decode_kernel(
         dtype_code(dtype), batch, q_heads, kv_heads, head_dim, block_size, max_seq_len, total_seq_len,
         _array_ptr(lens), int(device_planned))]
+
+
+PREFILL_ORDERS = ("none", "table", "sorted", "requests")
+
+
+def prefill_order(query_lens, context_lens, q_heads: int, kv_heads: int, head_dim: int, host_plan: bool = True) -> str:
+    """Where a prefill call's workgroups take their query tiles from ("none": not on the MFMA kernels)."""
+    cu, ctx = _host_lengths(np.concatenate([[0], np.cumsum(query_lens)]), context_lens, len(query_lens))
+    ends = [c + n for c, n in zip(context_lens, query_lens)]
+    return PREFILL_ORDERS[load_library().nie_varlen_prefill_order(
+        len(query_lens), sum(query_lens), max(query_lens), max(ends), q_heads, kv_heads, head_dim,
+        _array_ptr(cu) if host_plan else None, _array_ptr(ctx) if host_plan else None)]
 
 
 def _check(rc: int, what: str) -> None:
