@@ -294,12 +294,12 @@ int nie_attention_rounding(void);
  * instead of the two pass launches and the sum of their split partials: each
  * split keeps its scores on chip, the splits exchange only their (max, sum)
  * pairs and output shares, through counters and records in the workspace's
- * control region, and the split that finishes last sums the shares.  A call
- * planned on the host (host lengths, or a device-resident plan) does so at
- * head_dim 64 and 128 with GQA groups up to 16 while a split's scores fit
- * (32 tiles at 4 query heads per KV head of 64); any call at head_dim 64 with
- * groups of at most 4 query heads.  nie_set_decode_fused(0)
- * turns it off for calls issued after it in the whole process (1, the
+ * control region, and the split that finishes last sums the shares.  Any call
+ * does so at head_dim 64 with groups of at most 4 query heads; a call planned
+ * on the host at head_dim 64 and 128 with GQA groups up to 16 where that is
+ * the faster way and a split's scores fit (nie_paged_decode_kernel tells), and
+ * a call with a device-resident plan where that holds for every plan within
+ * its bounds.  nie_set_decode_fused(0) turns it off for calls issued after it in the whole process (1, the
  * default, on); the pass launches then run the same plan, so both give the
  * same bits.  The switch also covers the one-pass rounding (fp32, and bf16
  * with NIE_ROUND_FAST): there, when a call splits its sequences' keys, the
@@ -532,7 +532,9 @@ int nie_paged_decode_append_planned(int dtype,
  * of the same arguments above the maximum, for a call that splits) returns
  * NIE_EINVAL with a message saying so.  All calls on one GPU share the
  * array: calls that overlap in time on one GPU (different streams, or
- * different threads) race.  Nothing in the array needs clearing between
+ * different threads) race, whatever their shape (a GQA group outside {1, 2, 4,
+ * 8, 16} uses it when its partials fit, and runs on the generic kernel
+ * otherwise).  Nothing in the array needs clearing between
  * calls (each call writes every partial it reads).
  * No counterpart in the reference: this entry point exists for callers that
  * cannot allocate device memory — code under HIP graph capture, tight
